@@ -103,17 +103,6 @@ int32_t gated_width(const mlora_int4_t* w, int32_t flags) {
 // The residual epilogue (MLORA_EPILOGUE_RESIDUAL): y holds the residual and receives residual + output.
 bool residual_of(int32_t flags) { return (flags & MLORA_EPILOGUE_RESIDUAL) != 0; }
 
-// CUs of the current device (256 when it cannot be asked, e.g. on a host without a GPU).
-int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cus[dev] == 0 && (hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-                        cus[dev] <= 0))
-    cus[dev] = 256;
-  return cus[dev];
-}
-
 int base_of(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* r, int64_t x_stride, int32_t flags,
             Base* out) {
   const bool gated = (flags & MLORA_EPILOGUE_SILU_MUL) != 0, resid = residual_of(flags);
@@ -212,6 +201,40 @@ size_t partials_of(const mlora_int4_t* w, const mlora_route_t* r, Base base, int
   return base == Base::split ? split_bytes(w, r->tokens) : 0;
 }
 
+// Whether a product of the family `base` runs as a sliced product (sliced.hip) instead of the family's own kernels. The
+// rule reads shapes only, never the epilogue, so a group's plain, gated and residual products sum in one order.
+//  - fused, long segments: when its estimate is below the 256 x 256 tiles' (a round of at most half the CUs: 19 us and
+//    0.94 a step; fuller: 1.4 a step), e.g. 384 rows of 2048 -> 2048, 6144 -> 2048 and 2048 -> 12288: 13, 24 and 38 us
+//    against 45, 101 and 48; 2311 rows of 2048 -> 12288 stay on the tiles (131 us against 178);
+//  - split (short segments, 257 to 1023 rows): its segments' second factors in turn take about 1.8 us each, shared by the
+//    input slices, against the split product's range launch and epilogue: 643 rows of 128 adapters, 2048 -> 4096 and
+//    2048: 36 and 26 us against 46 and 40, 6144 -> 2048 equal, 2048 -> 12288 100 against 85;
+//  - narrow: at most 32 rows whose columns alone fill the CUs (one input range: 2048 -> 12288 12 us against 26).
+bool use_slice(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* r, int64_t x_stride, Base base,
+               int32_t flags) {
+  const int32_t forced = (flags >> 8) & 0xF;
+  if (base == Base::gemv || forced > 1 || r->tokens == 0 || L->rank_cap > MLORA_SPLIT_MAX_RANK) return false;
+  const int64_t row = x_stride > w->k ? x_stride : w->k;
+  if (row >= ((int64_t)1 << 31) / r->tokens) return false;
+  if (base == Base::narrow) return r->tokens <= 32 && narrow_ranges(w, flags) == 1;
+  double us = 0.0;
+  const SliceForm f = slice_form(r->tokens, w->columns, w->k, &us);
+  const int64_t cus = device_cus(), steps = w->k / 64;
+  if (base == Base::fused) {
+    if (!long_segments(r, L->pool_rows)) return false;
+    const int64_t tiles = ((r->tokens + 255) / 256) * ((w->columns + 255) / 256);
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    return us < (double)rounds * (19.0 + (2 * tiles <= cus ? 0.94 : 1.4) * (double)steps);
+  }
+  const int64_t segs = r->requests < L->pool_rows ? r->requests : L->pool_rows;
+  const int64_t wgs = ((r->tokens + 32 * f.rb - 1) / (32 * f.rb)) * ((w->columns / 64 + f.cw - 1) / f.cw);
+  const double in_tile = (double)(32 * f.rb) * (double)segs / (double)r->tokens + 1.0;
+  us += 1.8 * (double)((wgs + cus - 1) / cus) * in_tile / f.kw;
+  const int64_t ranges = split_ranges(w, r->tokens);
+  const int64_t tiles = ((r->tokens + 255) / 256) * ((w->columns + 255) / 256) * ranges;
+  return us < (double)((tiles + cus - 1) / cus) * (14.0 + 1.1 * (double)(steps / ranges)) + 14.0 +
+                  (double)w->columns * (double)r->tokens * 3.0e-6;
+}
 // The base product and the LoRA second factor once mid holds the first factors, or, for a narrow product with
 // fuse_shrink, as it computes them (its base launch writes mid).
 int run_base(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* r, const uint16_t* x,
@@ -219,6 +242,13 @@ int run_base(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* 
              void* partials, size_t partials_bytes, Base base, int32_t flags, hipStream_t s) {
   const int32_t inter = gated_width(w, flags);
   const bool resid = residual_of(flags);
+  if (use_slice(w, L, r, x_stride, base, flags)) {
+    if (fuse_shrink) {
+      const int rc = launch_shrink(*L, *r, x, x_stride, w->k, mid, false, s);
+      if (rc) return rc;
+    }
+    return launch_slice(*w, *L, *r, x, x_stride, y, y_stride, last_out, w->out, mid, s, inter, resid);
+  }
   if (base == Base::narrow) {
     const int32_t ks = narrow_ranges(w, flags);
     const size_t need = dec_partials_bytes(*w, ks);
@@ -256,6 +286,16 @@ uint8_t* noalloc_scratch() {
 }
 
 }  // namespace
+
+int device_cus() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cus[dev] == 0 && (hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+                        cus[dev] <= 0))
+    cus[dev] = 256;
+  return cus[dev];
+}
 
 #pragma GCC visibility push(default)
 extern "C" {
@@ -391,12 +431,13 @@ int mlora_int4_linear(const mlora_int4_t* w, const mlora_lora_t* lora, const mlo
   if (workspace_bytes < mlora_workspace_bytes(route->tokens, lora->rank_cap)) return MLORA_EWORKSPACE;
   Base base;
   if ((rc = base_of(w, lora, route, x_stride, flags, &base))) return rc;
-  if (base == Base::split && (partials == nullptr || partials_bytes < split_bytes(w, route->tokens)))
+  const bool sliced = use_slice(w, lora, route, x_stride, base, flags);
+  if (base == Base::split && !sliced && (partials == nullptr || partials_bytes < split_bytes(w, route->tokens)))
     return MLORA_EWORKSPACE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint16_t* mid = static_cast<uint16_t*>(workspace);
   const bool mfma_shrink = shrink_on_mfma(route, lora->pool_rows, flags);
-  if (base == Base::split && !mfma_shrink) {
+  if (base == Base::split && !mfma_shrink && !sliced) {
     // split product of short segments: the first factor (its own launch: two of its workgroups fit a CU, where the
     // base launch's LDS leaves room for one), the base ranges, then the epilogue
     const int32_t ks = split_ranges(w, route->tokens);
@@ -407,7 +448,7 @@ int mlora_int4_linear(const mlora_int4_t* w, const mlora_lora_t* lora, const mlo
     return launch_finish(*lora, *route, part, ks, w->columns, mid, y, y_stride, last_out, w->out, s,
                          gated_width(w, flags), residual_of(flags));
   }
-  if (base == Base::split) {
+  if (base == Base::split && !sliced) {
     // split product of long segments (forced): the first factor, the base ranges, then the epilogue
     const int32_t ks = split_ranges(w, route->tokens);
     float* part = static_cast<float*>(partials);

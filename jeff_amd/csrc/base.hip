@@ -189,7 +189,6 @@ constexpr int kGvCols = 16, kGvSlices = 64;  // columns per workgroup; input sli
 constexpr int kGvMaxTokens = 8;
 constexpr int kGvChunk = 2048;               // inputs of x staged in LDS at a time (8 rows x 4 KB)
 constexpr int kGvRows = kGvChunk / 8 / kGvSlices;  // word rows per thread and chunk
-constexpr int kBigTileTokens = 1024;  // from here on the 256 x 256 tiles of gemm256.hip fill the chip
 
 static_assert(kGvSlices * kGvMaxTokens * kGvCols * 4 <= kGvMaxTokens * kGvChunk * 2, "the sums reuse the x buffer");
 
@@ -337,8 +336,9 @@ int launch_base(const mlora_int4_t* w, const mlora_lora_t& L, const mlora_route_
     else
       hipLaunchKernelGGL(base_gemv_kernel<false>, dim3(blocks), dim3(256), 0, stream, none, L, r, x, x_stride, y,
                          y_stride, last_out, n_out, mid);
-  } else if (w != nullptr && r.tokens >= kBigTileTokens && r.tokens * x_stride < ((int64_t)1 << 31)) {
-    // (the 256 x 256 kernel addresses x rows with 32-bit element offsets)
+  } else if (w != nullptr && r.tokens * x_stride < ((int64_t)1 << 31)) {
+    // the 256 x 256 tiles, which address x rows with 32-bit element offsets (base_mfma_kernel's base form takes the
+    // passes past them: 384 rows of 2048 -> 4096 took it 58 us, the tiles 49)
     return launch_base256(*w, L, r, x, x_stride, y, y_stride, last_out, n_out, mid, nullptr, 1, stream);
   } else {
     const int m_tiles = (int)((r.tokens + kBM - 1) / kBM);

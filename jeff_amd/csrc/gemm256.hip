@@ -706,20 +706,9 @@ __global__ __launch_bounds__(kThreads) void base_mfma256_kernel(mlora_int4_t w, 
 // its segments' sB rather than to its K loop) 128 rows when that is strictly fewer, e.g. 4096 decode rows through
 // 2048 columns: 128 tiles of 256 rows leave half the CUs idle. Split launches keep 256 (their range count is sized
 // for 256-row tiles).
-// The current device's compute units (0 if unknown), read once per device.
-static int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cus[dev] == 0 && hipDeviceGetAttribute(&cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    cus[dev] = 0;
-  return cus[dev] > 0 ? cus[dev] : 0;
-}
-
 int tile_blocks(int64_t tokens, int n_tiles, int32_t ksplit, bool short_segs) {
   if (ksplit != 1) return 8;
   const int cus = device_cus();
-  if (cus <= 0) return 8;
   auto cost = [&](int mb) {
     const int64_t tiles = ((tokens + 32 * mb - 1) / (32 * mb)) * n_tiles;
     return ((tiles + cus - 1) / cus) * mb;

@@ -35,15 +35,16 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 // 8-bit significand, and their difference has at most 13 significant bits, so the single rounding to bf16 is the
 // only one. zs = z * s is formed once per (group, column) by the caller.
 __device__ __forceinline__ uint4 dequant_word(uint32_t w, float s, float zs) {
-  uint32_t lo = w & 0x0F0F0F0Fu;         // codes of inputs 0, 2, 4, 6 in bytes 0..3
-  uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;  // codes of inputs 1, 3, 5, 7
-  // keep the byte layout visible to the compiler so each code converts with one v_cvt_f32_ubyteN
-  asm volatile("" : "+v"(lo));
-  asm volatile("" : "+v"(hi));
-  const float c0 = (float)(lo & 0xFF), c2 = (float)((lo >> 8) & 0xFF);
-  const float c4 = (float)((lo >> 16) & 0xFF), c6 = (float)(lo >> 24);
-  const float c1 = (float)(hi & 0xFF), c3 = (float)((hi >> 8) & 0xFF);
-  const float c5 = (float)((hi >> 16) & 0xFF), c7 = (float)(hi >> 24);
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  const uint32_t lo = w & 0x0F0F0F0Fu;         // codes of inputs 0, 2, 4, 6 in bytes 0..3
+  const uint32_t hi = (w >> 4) & 0x0F0F0F0Fu;  // codes of inputs 1, 3, 5, 7
+  // A code c in a byte is the e4m3 number c 2^-9 (denormal below 8, then linear on to 15), so one conversion scaled by
+  // 2^9 turns two codes into float32, where v_cvt_f32_ubyteN takes one at the same rate.
+  const f32x2_t c02 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, false);
+  const f32x2_t c46 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, true);
+  const f32x2_t c13 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, false);
+  const f32x2_t c57 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, true);
+  const float c0 = c02.x, c2 = c02.y, c4 = c46.x, c6 = c46.y, c1 = c13.x, c3 = c13.y, c5 = c57.x, c7 = c57.y;
   uint4 r;
   r.x = pack_bf16x2(__builtin_fmaf(c0, s, -zs), __builtin_fmaf(c1, s, -zs));
   r.y = pack_bf16x2(__builtin_fmaf(c2, s, -zs), __builtin_fmaf(c3, s, -zs));
@@ -253,3 +254,15 @@ int launch_dec(const mlora_int4_t& w, const mlora_lora_t& L, const mlora_route_t
 int launch_base(const mlora_int4_t* w, const mlora_lora_t& L, const mlora_route_t& r, const uint16_t* x,
                 int64_t x_stride, uint16_t* y, int64_t y_stride, uint16_t* last_out, int32_t n_out,
                 const uint16_t* mid, bool gemv, hipStream_t stream);
+// Compute units of the current device (256 when it cannot be asked, e.g. on a host without a GPU), read once per device.
+int device_cus();
+// A sliced product's tile (sliced.hip): rb row blocks of 32 by cw groups of 64 columns, the inputs in kw slices.
+struct SliceForm {
+  int rb, cw, kw;
+};
+SliceForm slice_form(int64_t tokens, int32_t columns, int32_t k, double* us);
+// Sliced product: one launch once mid holds the first factors (inter and residual as above; the group's columns a
+// multiple of 64, gated: inter a multiple of 32; tokens x max(x_stride, k) below 2^31).
+int launch_slice(const mlora_int4_t& w, const mlora_lora_t& L, const mlora_route_t& r, const uint16_t* x,
+                 int64_t x_stride, uint16_t* y, int64_t y_stride, uint16_t* last_out, int32_t n_out,
+                 const uint16_t* mid, hipStream_t stream, int32_t inter, bool residual);

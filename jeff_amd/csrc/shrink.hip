@@ -190,6 +190,105 @@ __global__ __launch_bounds__(256) void shrink_tile_kernel(mlora_lora_t L, mlora_
   }
 }
 
+// Long segments in a small or medium pass: one workgroup per (32 sorted rows, 32 stacked ranks), its 16 waves slicing
+// the inputs (wave w the 64-input chunks w, w + 16, ...), as slice_kernel (sliced.hip) slices the base product's: a
+// pass of few row tiles has few workgroups, and with all the inputs in one wave each would walk them in one long chain.
+// A wave stages its chunk's x rows and A rows in two LDS slots of its own (loads that write LDS directly, whole
+// 128-byte rows), takes the operands into registers, re-fills the slots and multiplies; there is no barrier before the
+// waves' sums are added in wave order. Segments crossing the rows are taken in turn.
+constexpr int kRowWaves = 16;
+__global__ __launch_bounds__(kRowWaves * 64) void shrink_rows_kernel(mlora_lora_t L, mlora_route_t r,
+                                                                    const uint16_t* __restrict__ x, int64_t x_stride,
+                                                                    int32_t k, uint16_t* __restrict__ mid) {
+  __shared__ __attribute__((aligned(16))) uint16_t w_x[kRowWaves * 32 * kSChunk];
+  __shared__ __attribute__((aligned(16))) uint16_t w_a[kRowWaves * 32 * kSChunk];
+  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T = (int)r.tokens, R = L.rank_cap;
+  const int p0 = (int)blockIdx.x * 32, p1 = min(p0 + 32, T), b0 = (int)blockIdx.y * 32;
+  // instruction i fills rows 8 i + (lane >> 3); lane l writes slot l & 7 of its row, which holds the row's 16-byte
+  // chunk swz_slot(row, l & 7); rows past the pass re-read its last row, ranks past the stack the last rank
+  const uint16_t* xsrc[4];
+  int aoff[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    xsrc[i] = x + (int64_t)r.tok_perm[min(p0 + row, T - 1)] * x_stride + 8 * swz_slot(row, lane & 7);
+    aoff[i] = min(row, R - 1 - b0) * k + 8 * swz_slot(row, lane & 7);
+  }
+  const int nk = k / kSChunk;
+  const int n = wave < nk ? (nk - wave + kRowWaves - 1) / kRowWaves : 0;
+  const int s_lo = r.seg_of[p0], s_hi = r.seg_of[p1 - 1];
+  for (int s = s_lo; s <= s_hi; ++s) {
+    const int a = r.seg_adapter[s];
+    if (a == 0) continue;  // the base row: no first factor
+    const int sb = r.seg_start[s], se = r.seg_start[s + 1];
+    bool any = false;  // the adapter has a live rank in this block
+    for (int j = 0, rho = 0; j < L.n_mats; rho += L.cap[j++])
+      any = any || (rho < b0 + 32 && rho + live_rank(L, a, j) > b0);
+    if (!any) continue;
+    const uint16_t* Ablk = L.pool + (int64_t)a * L.pool_stride + L.off_a + (int64_t)b0 * k;
+    auto issue = [&](int i) __attribute__((always_inline)) {
+      const int kc = (wave + kRowWaves * i) * kSChunk;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        __builtin_amdgcn_global_load_lds(xsrc[q] + kc, (lds_void*)(w_x + (wave * 32 + q * 8) * kSChunk), 16, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        __builtin_amdgcn_global_load_lds(Ablk + aoff[q] + kc, (lds_void*)(w_a + (wave * 32 + q * 8) * kSChunk), 16, 0,
+                                         0);
+    };
+    f32x16_t acc = f32x16_t{};
+    if (n > 0) issue(0);
+    for (int i = 0; i < n; ++i) {
+      uint4 xv[4], av[4];
+      const uint4* xs = reinterpret_cast<const uint4*>(w_x);
+      const uint4* as = reinterpret_cast<const uint4*>(w_a);
+      MLORA_WAIT_VM(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int at = (wave * 32 * kSChunk + swz(lane & 31, 2 * u + h)) >> 3;
+        xv[u] = xs[at];
+        av[u] = as[at];
+      }
+      drain_lds();  // the slots' reads are done
+      if (i + 1 < n) issue(i + 1);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = mfma32(av[u], xv[u], acc);
+    }
+    // lane l holds row p0 + (l & 31), stacked ranks b0 + 8 g + 4 (l >> 5) + e: the waves' sums added in wave order
+    float4* red = reinterpret_cast<float4*>(w_x);
+    __syncthreads();  // every wave is done with its slots
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      red[(wave * 4 + g) * 64 + lane] = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+    __syncthreads();
+    if (tid < 256) {
+      float4 v = red[tid];
+#pragma unroll
+      for (int q = 1; q < kRowWaves; ++q) {
+        const float4 t = red[q * 256 + tid];
+        v.x += t.x, v.y += t.y, v.z += t.z, v.w += t.w;
+      }
+      const int p = p0 + (lane & 31), n0 = b0 + 8 * wave + 4 * h;
+      if (p >= sb && p < se && p < T && n0 < R) {
+        int j = 0, rho = 0;  // the matrix holding rank n0 (capacities are multiples of 8: n0 .. n0 + 3 share it)
+        while (j + 1 < L.n_mats && n0 >= rho + L.cap[j]) rho += L.cap[j++];
+        const int live = live_rank(L, a, j) - (n0 - rho);
+        uint16_t* mrow = mid + (int64_t)p * R + n0;
+        const uint32_t lo = pack_bf16x2(v.x, v.y), hi = pack_bf16x2(v.z, v.w);
+        if (live >= 4) {
+          *reinterpret_cast<uint2*>(mrow) = make_uint2(lo, hi);
+        } else {
+          const uint16_t o[4] = {(uint16_t)lo, (uint16_t)(lo >> 16), (uint16_t)hi, (uint16_t)(hi >> 16)};
+          for (int e = 0; e < live; ++e) mrow[e] = o[e];
+        }
+      }
+    }
+    __syncthreads();  // the sums are read before the next segment's slots are filled
+  }
+}
+
 // Short segments (decode): one workgroup per (segment, 32-rank block), the body in shrink_seg.h.
 __global__ __launch_bounds__(kDWaves * 64) void shrink_seg_kernel(mlora_lora_t L, mlora_route_t r,
                                                                  const uint16_t* __restrict__ x, int64_t x_stride,
@@ -208,6 +307,17 @@ int launch_shrink(const mlora_lora_t& L, const mlora_route_t& r, const uint16_t*
     // 32-rank blocks of the stacked capacity, in passes of at most 4 (as even as the count allows)
     const int nblk = (L.rank_cap + 31) / 32;
     if (nblk == 0) return MLORA_OK;
+    // Rows of 32 with the inputs sliced over 16 waves, where its estimate (a workgroup a CU: 9 us a round and one per
+    // chunk of a wave) is below the 128-row tiles' (their waves walk every chunk: 5.5 us and 0.335 a chunk). 2311 rows,
+    // K 2048 and 6144: 13 and 16 us against 22 and 34; 32 rows: 5 to 7 against 12 to 37; 8855 rows, K 1024: the tiles,
+    // 10 us against 12.
+    const int64_t wgs = (r.tokens + 31) / 32 * nblk, nk = k / kSChunk;
+    if ((double)((wgs + device_cus() - 1) / device_cus()) * (9.0 + (double)((nk + kRowWaves - 1) / kRowWaves)) <
+        5.5 + 0.335 * (double)nk) {
+      const dim3 rows((unsigned)((r.tokens + 31) / 32), (unsigned)nblk);
+      hipLaunchKernelGGL(shrink_rows_kernel, rows, dim3(kRowWaves * 64), 0, stream, L, r, x, x_stride, k, mid);
+      return hipGetLastError() == hipSuccess ? MLORA_OK : MLORA_ELAUNCH;
+    }
     const int passes = (nblk + 3) / 4, rb = (nblk + passes - 1) / passes;
     const dim3 grid((unsigned)((r.tokens + 127) / 128), 2);
     // ring slots: 20 KB a slot at one block (4 slots, two workgroups per CU), 24 KB at two (3 slots, two per CU),
