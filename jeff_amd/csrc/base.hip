@@ -68,7 +68,6 @@ __device__ __forceinline__ void expand_into(f32x16_t (&acc)[2][2], int64_t prow,
   }
 }
 
-template <bool kBase>
 __global__ __launch_bounds__(256) void base_mfma_kernel(mlora_int4_t w, mlora_lora_t L, mlora_route_t r,
                                                        const uint16_t* __restrict__ x, int64_t x_stride,
                                                        uint16_t* __restrict__ y, int64_t y_stride,
@@ -88,58 +87,56 @@ __global__ __launch_bounds__(256) void base_mfma_kernel(mlora_int4_t w, mlora_lo
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = f32x16_t{};
 
-  if constexpr (kBase) {
-    const int xr = tid >> 1, xh = (tid & 1) * 32;  // x staging: 32 inputs of one row per thread
-    const int64_t xp = p0 + xr;
-    const uint16_t* xsrc = xp < T ? x + (int64_t)r.tok_perm[xp] * x_stride + xh : nullptr;
-    const int wc = tid & (kBN - 1), wr0 = (tid >> 7) * 4;  // weight staging: 4 words (32 inputs) of one column
-    const int col = n0 + wc;
-    const bool colok = col < w.columns;
-    uint4 xreg[4];
-    uint32_t wreg[4];
-    float sc = 1.0f, zsc = 8.0f;
-    auto fetch = [&](int kc) {
+  const int xr = tid >> 1, xh = (tid & 1) * 32;  // x staging: 32 inputs of one row per thread
+  const int64_t xp = p0 + xr;
+  const uint16_t* xsrc = xp < T ? x + (int64_t)r.tok_perm[xp] * x_stride + xh : nullptr;
+  const int wc = tid & (kBN - 1), wr0 = (tid >> 7) * 4;  // weight staging: 4 words (32 inputs) of one column
+  const int col = n0 + wc;
+  const bool colok = col < w.columns;
+  uint4 xreg[4];
+  uint32_t wreg[4];
+  float sc = 1.0f, zsc = 8.0f;
+  auto fetch = [&](int kc) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        xreg[i] = xsrc != nullptr ? *reinterpret_cast<const uint4*>(xsrc + kc + 8 * i) : make_uint4(0, 0, 0, 0);
-      if (colok) {
+    for (int i = 0; i < 4; ++i)
+      xreg[i] = xsrc != nullptr ? *reinterpret_cast<const uint4*>(xsrc + kc + 8 * i) : make_uint4(0, 0, 0, 0);
+    if (colok) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wreg[i] = (uint32_t)w.words[(int64_t)(kc / 8 + wr0 + i) * w.columns + col];
-        const int64_t g = (int64_t)(kc / w.group) * w.columns + col;
-        sc = bf16_to_f32(w.scales[g]);
-        zsc = (w.zeros != nullptr ? (float)w.zeros[g] : 8.0f) * sc;
-      } else {
+      for (int i = 0; i < 4; ++i) wreg[i] = (uint32_t)w.words[(int64_t)(kc / 8 + wr0 + i) * w.columns + col];
+      const int64_t g = (int64_t)(kc / w.group) * w.columns + col;
+      sc = bf16_to_f32(w.scales[g]);
+      zsc = (w.zeros != nullptr ? (float)w.zeros[g] : 8.0f) * sc;
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wreg[i] = 0x88888888u;  // columns past the layout: zero weights
-        sc = 1.0f;
-        zsc = 8.0f;
-      }
-    };
-    fetch(0);
-    for (int kc = 0; kc < w.k; kc += kBK) {
-      __syncthreads();  // the previous step's MFMAs are done with the LDS tiles
+      for (int i = 0; i < 4; ++i) wreg[i] = 0x88888888u;  // columns past the layout: zero weights
+      sc = 1.0f;
+      zsc = 8.0f;
+    }
+  };
+  fetch(0);
+  for (int kc = 0; kc < w.k; kc += kBK) {
+    __syncthreads();  // the previous step's MFMAs are done with the LDS tiles
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&xs[xr * kLd + xh + 8 * i]) = xreg[i];
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&xs[xr * kLd + xh + 8 * i]) = xreg[i];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<uint4*>(&wsm[wc * kLd + (wr0 + i) * 8]) = dequant_word(wreg[i], sc, zsc);
-      __syncthreads();
-      if (kc + kBK < w.k) fetch(kc + kBK);
+    for (int i = 0; i < 4; ++i)
+      *reinterpret_cast<uint4*>(&wsm[wc * kLd + (wr0 + i) * 8]) = dequant_word(wreg[i], sc, zsc);
+    __syncthreads();
+    if (kc + kBK < w.k) fetch(kc + kBK);
 #pragma unroll
-      for (int k16 = 0; k16 < kBK / 16; ++k16) {
-        const int kk = k16 * 16 + (lane >> 5) * 8;
-        uint4 a[2], b[2];
+    for (int k16 = 0; k16 < kBK / 16; ++k16) {
+      const int kk = k16 * 16 + (lane >> 5) * 8;
+      uint4 a[2], b[2];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
-          a[mb] = *reinterpret_cast<const uint4*>(&xs[(wm * 64 + mb * 32 + (lane & 31)) * kLd + kk]);
+      for (int mb = 0; mb < 2; ++mb)
+        a[mb] = *reinterpret_cast<const uint4*>(&xs[(wm * 64 + mb * 32 + (lane & 31)) * kLd + kk]);
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-          b[nb] = *reinterpret_cast<const uint4*>(&wsm[(wn * 64 + nb * 32 + (lane & 31)) * kLd + kk]);
+      for (int nb = 0; nb < 2; ++nb)
+        b[nb] = *reinterpret_cast<const uint4*>(&wsm[(wn * 64 + nb * 32 + (lane & 31)) * kLd + kk]);
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = mfma32(a[mb], b[nb], acc[mb][nb]);
-      }
+        for (int nb = 0; nb < 2; ++nb) acc[mb][nb] = mfma32(a[mb], b[nb], acc[mb][nb]);
     }
   }
 
@@ -153,17 +150,6 @@ __global__ __launch_bounds__(256) void base_mfma_kernel(mlora_int4_t w, mlora_lo
       const int64_t p = prow + mb * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
       orig[mb][i] = p < T ? r.tok_perm[p] : -1;
     }
-  if constexpr (!kBase) {  // lora_add: start from y
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
-        const int c = pcol + nb * 32 + (lane & 31);
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (orig[mb][i] >= 0 && c < n_out) acc[mb][nb][i] = bf16_to_f32(y[(int64_t)orig[mb][i] * y_stride + c]);
-      }
-  }
   expand_into(acc, prow, pcol, L, r, mid, n_out, lane);
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
@@ -183,6 +169,113 @@ __global__ __launch_bounds__(256) void base_mfma_kernel(mlora_int4_t w, mlora_lo
         }
       }
     }
+}
+
+// lora_add over more than 8 tokens: y += mid sB in place, a stream over y (read once, written once) with a short product
+// beside it. A workgroup takes 64 sorted rows x 128 columns; its y rows are asked for first, whole 256-byte pieces; each of
+// its 4 waves sums the LoRA term of 32 columns by MFMA over the segments crossing the rows, in float32; the tile then
+// goes through LDS into row order, where it is added to y and rounded once. 4501 rows x 12288 columns of bf16: 243 us
+// when y was read and written by the MFMA layout's lanes (2 bytes of 32 columns a time).
+constexpr int kAddRows = 64, kAddCols = 128, kAddPitch = kAddCols + 4;  // (rows 528 bytes apart: 16 rows on all banks)
+
+__global__ __launch_bounds__(256) void lora_add_kernel(mlora_lora_t L, mlora_route_t r, uint16_t* __restrict__ y,
+                                                       int64_t y_stride, int32_t n_out,
+                                                       const uint16_t* __restrict__ mid, int32_t n_tiles, int32_t vec) {
+  __shared__ __attribute__((aligned(16))) float tile[kAddRows * kAddPitch];
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int T = (int)r.tokens;
+  const int mt = blockIdx.x / n_tiles, nt = blockIdx.x - mt * n_tiles;
+  const int p0 = mt * kAddRows, p1 = min(p0 + kAddRows, T);
+  const int n0 = nt * kAddCols;
+  // the thread's pieces of y: rows (tid / 16) + 16 q, columns n0 + 8 (tid % 16) .. +7
+  const int ycol = n0 + 8 * (tid & 15);
+  int64_t yoff[4];
+  uint4 yv[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int p = p0 + 16 * q + (tid >> 4);
+    yoff[q] = p < T && ycol < n_out ? (int64_t)r.tok_perm[p] * y_stride + ycol : -1;
+  }
+  const bool whole = vec && ycol + 7 < n_out;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (whole && yoff[q] >= 0) yv[q] = *reinterpret_cast<const uint4*>(y + yoff[q]);
+  f32x16_t acc[2] = {f32x16_t{}, f32x16_t{}};
+  const int c0 = n0 + wave * 32;
+  if (c0 < n_out) {
+    const int s_lo = r.seg_of[p0], s_hi = r.seg_of[p1 - 1];
+    const int jlo = matrix_of(L, c0), jhi = matrix_of(L, min(c0 + 31, n_out - 1));
+    for (int t0 = s_lo; t0 <= s_hi; t0 += kWave) {
+      // lane i: segment t0 + i's adapter and bounds relative to the tile
+      const int cnt = min(kWave, s_hi - t0 + 1), s = t0 + min(lane, cnt - 1);
+      const int ta = r.seg_adapter[s], tb = r.seg_start[s] - p0, te = r.seg_start[s + 1] - p0;
+      for (int j = jlo; j <= jhi; ++j) {
+        const int tl = ta == 0 ? 0 : live_rank(L, ta, j);  // row 0 is the base: no update
+        const int oj = col_offset(L, j), rho = rank_offset(L, j), cc = c0 + li - oj;
+        const bool cin = cc >= 0 && cc < L.cols[j] && c0 + li < n_out;
+        for (int i = 0; i < cnt; ++i) {
+          const int rank = __builtin_amdgcn_readlane(tl, i);
+          if (rank == 0) continue;
+          const int a = __builtin_amdgcn_readlane(ta, i);
+          const int sb = __builtin_amdgcn_readlane(tb, i), se = __builtin_amdgcn_readlane(te, i);
+          const uint16_t* brow = L.pool + (int64_t)a * L.pool_stride + L.off_b[j] +
+                                 (int64_t)(cin ? cc : 0) * sb_stride(rank, L.cap[j]) + 8 * h;
+          for (int k0 = 0; k0 < rank; k0 += 32) {
+            uint4 bv[2], av[2][2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              const int kk = k0 + 16 * u, left = rank - kk - 8 * h;  // live ranks of the lane's eight
+              bv[u] = cin && left > 0 ? keep_first(*reinterpret_cast<const uint4*>(brow + kk), left)
+                                      : make_uint4(0, 0, 0, 0);
+#pragma unroll
+              for (int mb = 0; mb < 2; ++mb) {
+                const int row = mb * 32 + li;
+                av[mb][u] = row >= sb && row < se && left > 0
+                                ? keep_first(*reinterpret_cast<const uint4*>(mid + (int64_t)(p0 + row) * L.rank_cap + rho +
+                                                                             kk + 8 * h),
+                                             left)
+                                : make_uint4(0, 0, 0, 0);
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              if (k0 + 16 * u >= rank) break;
+#pragma unroll
+              for (int mb = 0; mb < 2; ++mb)
+                if (mb * 32 < se && mb * 32 + 32 > sb) acc[mb] = mfma32(bv[u], av[mb][u], acc[mb]);
+            }
+          }
+        }
+      }
+    }
+  }
+  // lane l holds row 32 mb + (l & 31), columns 8 g + 4 (l >> 5) .. +3 of the wave's 32
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<float4*>(&tile[(mb * 32 + li) * kAddPitch + wave * 32 + 8 * g + 4 * h]) =
+          make_float4(acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (yoff[q] < 0) continue;
+    const float* t = &tile[(16 * q + (tid >> 4)) * kAddPitch + 8 * (tid & 15)];
+    const float4 lo = *reinterpret_cast<const float4*>(t), hi = *reinterpret_cast<const float4*>(t + 4);
+    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    if (whole) {
+      const uint32_t yw[4] = {yv[q].x, yv[q].y, yv[q].z, yv[q].w};
+      uint32_t o[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = pack_bf16x2(bf16_lo(yw[e]) + v[2 * e], bf16_hi(yw[e]) + v[2 * e + 1]);
+      *reinterpret_cast<uint4*>(y + yoff[q]) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (ycol + e < n_out) y[yoff[q] + e] = f32_to_bf16(bf16_to_f32(y[yoff[q] + e]) + v[e]);
+    }
+  }
 }
 
 constexpr int kGvCols = 16, kGvSlices = 64;  // columns per workgroup; input slices (4 columns x 64 slices = 256 threads)
@@ -340,16 +433,17 @@ int launch_base(const mlora_int4_t* w, const mlora_lora_t& L, const mlora_route_
     // the 256 x 256 tiles, which address x rows with 32-bit element offsets (base_mfma_kernel's base form takes the
     // passes past them: 384 rows of 2048 -> 4096 took it 58 us, the tiles 49)
     return launch_base256(*w, L, r, x, x_stride, y, y_stride, last_out, n_out, mid, nullptr, 1, stream);
-  } else {
+  } else if (w != nullptr) {
     const int m_tiles = (int)((r.tokens + kBM - 1) / kBM);
-    const int n_tiles = (n_out + kBN - 1) / kBN;
-    const int64_t blocks = (int64_t)m_tiles * n_tiles;
-    if (w != nullptr)
-      hipLaunchKernelGGL(base_mfma_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, *w, L, r, x, x_stride,
-                         y, y_stride, last_out, n_out, mid, m_tiles);
-    else
-      hipLaunchKernelGGL(base_mfma_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, none, L, r, x,
-                         x_stride, y, y_stride, last_out, n_out, mid, m_tiles);
+    const int64_t blocks = (int64_t)m_tiles * ((n_out + kBN - 1) / kBN);
+    hipLaunchKernelGGL(base_mfma_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, *w, L, r, x, x_stride, y,
+                       y_stride, last_out, n_out, mid, m_tiles);
+  } else {
+    const int n_tiles = (n_out + kAddCols - 1) / kAddCols;
+    const int64_t blocks = (r.tokens + kAddRows - 1) / kAddRows * n_tiles;
+    const int32_t vec = reinterpret_cast<uintptr_t>(y) % 16 == 0 && y_stride % 8 == 0;  // 16-byte pieces of y
+    hipLaunchKernelGGL(lora_add_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, L, r, y, y_stride, n_out, mid,
+                       n_tiles, vec);
   }
   return hipGetLastError() == hipSuccess ? MLORA_OK : MLORA_ELAUNCH;
 }
