@@ -1,9 +1,12 @@
 // The decision head after the last projection: each request row's option logits from its own adapter's readout, then
 // the masked, tempered softmax (the reference's readout_rows: engine/batched_kernels.py:492-559, with
 // DecisionModel.forward's mask and temperature).
-//  - readout_logits_kernel: one workgroup per (row, 64 options); each wave takes 16 options, a lane 16-byte chunks of
-//    the hidden vector and of each option's readout row (coalesced across the wave), v_dot2_f32_bf16 into a float32
-//    partial, then a fixed shuffle tree across the wave; the sum is rounded to bf16 and stored as float32.
+//  - readout_logits_kernel: one workgroup per (up to 16 rows of one adapter, 64 options), so a readout is read once for
+//    16 of its requests. Its 4 waves slice the hidden dimension (32 inputs in turn); a wave multiplies 4 blocks of 16
+//    readout rows by the 16 hidden vectors with 16x16x32 bf16 MFMAs, operands straight from memory (16 rows of 64 bytes an
+//    instruction), and the waves' float32 sums are added in wave order, rounded to bf16 and stored as float32. Bound by
+//    the readouts' bytes: when every row read its own copy and each logit took a shuffle tree, 512 rows over 128 adapters
+//    took 64 us (0.5 GB through the caches, a chain of six lane exchanges a logit).
 //  - option_softmax_kernel: one wave per row; options from the row's count on get the logit -1e9, the logits are
 //    divided by the adapter's temperature and the softmax taken over all options (max and sum by fixed shuffle trees).
 #include "mlora_common.h"
@@ -13,10 +16,12 @@ namespace {
 using namespace mlora;
 
 constexpr int kRoOptionsPerBlock = 64;
-constexpr int kRoOptionsPerWave = 16;
 constexpr int kRoThreads = 256;
-constexpr int kRoGroup = 4;        // options whose readout loads are in flight together
-constexpr int kRoMaxChunks = 4;    // 16-byte chunks of the hidden vector per lane: dim <= 64 * 8 * 4 = 2048
+constexpr int kRoWaves = kRoThreads / 64;
+constexpr int kRoBlocks = kRoOptionsPerBlock / 16;  // 16-option MFMA blocks a wave takes
+constexpr int kRoRows = 16;                         // rows of one adapter a workgroup takes
+constexpr int kRoWindow = 1024;                     // ... among this many consecutive rows
+constexpr int kRoAhead = 4;                         // steps whose loads are in flight together
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -35,44 +40,82 @@ __global__ __launch_bounds__(kRoThreads) void readout_logits_kernel(const uint16
                                                                    const uint16_t* __restrict__ pool,
                                                                    int64_t pool_stride, int32_t options,
                                                                    int32_t pool_rows,
-                                                                   const int32_t* __restrict__ adapters,
+                                                                   const int32_t* __restrict__ adapters, int32_t rows,
                                                                    float* __restrict__ logits) {
-  const int b = blockIdx.x;
+  __shared__ float red[kRoWaves][kRoBlocks][4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int a = adapters[b];
-  if (a < 0 || a >= pool_rows) a = 0;  // an index outside the pool reads row 0: every read stays inside the pool
-  const uint16_t* h = hidden + (int64_t)b * hidden_stride;
-  const uint16_t* w = pool + (int64_t)a * pool_stride;
-  const int chunks = dim / 8;  // 16-byte chunks of a row; lane l takes chunks l, l + 64, ...
-  uint4 hv[kRoMaxChunks];
-#pragma unroll
-  for (int j = 0; j < kRoMaxChunks; ++j) {
-    const int c = lane + 64 * j;
-    hv[j] = c < chunks ? *reinterpret_cast<const uint4*>(h + 8 * c) : make_uint4(0, 0, 0, 0);
+  auto adapter_of = [&](int i) {
+    const int a = adapters[i];
+    return a < 0 || a >= pool_rows ? 0 : a;  // an index outside the pool reads row 0: every read stays inside the pool
+  };
+  // Block b leads if the rows of its adapter before it in its window are a multiple of 16; it then takes itself and the
+  // adapter's next 15 rows of the window, lane l the row l & 15 (past the last: its own again, never stored).
+  const int b = blockIdx.x;
+  const int a = adapter_of(b);
+  const int w0 = b - b % kRoWindow, w1 = min(w0 + kRoWindow, rows);
+  int before = 0;
+  for (int i = w0; i < b; i += 64) {
+    const int j = i + lane;
+    before += __popcll(__ballot(j < b && adapter_of(min(j, rows - 1)) == a));
   }
-  const int o0 = blockIdx.y * kRoOptionsPerBlock + wave * kRoOptionsPerWave;
-  for (int g = 0; g < kRoOptionsPerWave; g += kRoGroup) {
-    uint4 wv[kRoGroup][kRoMaxChunks];
+  if (before % kRoRows != 0) return;
+  int row = b, n = 1;
+  for (int i = b + 1; i < w1 && n < kRoRows; i += 64) {
+    const int j = i + lane;
+    uint64_t m = __ballot(j < w1 && adapter_of(min(j, rows - 1)) == a);
+    while (m != 0 && n < kRoRows) {
+      if ((lane & 15) == n) row = i + __ffsll((unsigned long long)m) - 1;
+      ++n;
+      m &= m - 1;
+    }
+  }
+  // operands: lane l holds row (option or request) l & 15, inputs 32 step + 8 (l >> 4) .. +7; options past the last re-read
+  // it (their sums are not stored), inputs past the dimension are zero
+  const int o0 = blockIdx.y * kRoOptionsPerBlock;
+  const uint16_t* hrow = hidden + (int64_t)row * hidden_stride + 8 * (lane >> 4);
+  const uint16_t* wrow[kRoBlocks];
 #pragma unroll
-    for (int i = 0; i < kRoGroup; ++i) {
-      const int o = min(o0 + g + i, options - 1);  // options past the last re-read it; their sums are not stored
+  for (int q = 0; q < kRoBlocks; ++q)
+    wrow[q] = pool + (int64_t)a * pool_stride + (int64_t)min(o0 + 16 * q + (lane & 15), options - 1) * dim + 8 * (lane >> 4);
+  f32x4_t acc[kRoBlocks];
 #pragma unroll
-      for (int j = 0; j < kRoMaxChunks; ++j) {
-        const int c = lane + 64 * j;
-        wv[i][j] = c < chunks ? *reinterpret_cast<const uint4*>(w + (int64_t)o * dim + 8 * c) : make_uint4(0, 0, 0, 0);
-      }
+  for (int q = 0; q < kRoBlocks; ++q) acc[q] = f32x4_t{};
+  const int steps = (dim + 31) / 32;
+  for (int s0 = wave; s0 < steps; s0 += kRoWaves * kRoAhead) {
+    uint4 hv[kRoAhead], wv[kRoAhead][kRoBlocks];
+#pragma unroll
+    for (int i = 0; i < kRoAhead; ++i) {
+      const int c = 32 * (s0 + kRoWaves * i);
+      const bool in = c + 8 * (lane >> 4) < dim;
+      hv[i] = in ? *reinterpret_cast<const uint4*>(hrow + c) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < kRoBlocks; ++q)
+        wv[i][q] = in ? *reinterpret_cast<const uint4*>(wrow[q] + c) : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < kRoGroup; ++i) {
-      float acc = 0.0f;
+    for (int i = 0; i < kRoAhead; ++i)
 #pragma unroll
-      for (int j = 0; j < kRoMaxChunks; ++j) acc = dot8(wv[i][j], hv[j], acc);
-      acc = wave_sum(acc);
-      const int o = o0 + g + i;
-      if (lane == 0 && o < options) logits[(int64_t)b * options + o] = bf16_to_f32(f32_to_bf16(acc));
-    }
+      for (int q = 0; q < kRoBlocks; ++q)
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wv[i][q]), as_bf16x8(hv[i]), acc[q], 0, 0, 0);
+  }
+  // lane l holds request l & 15, options 16 q + 4 (l >> 4) + e
+#pragma unroll
+  for (int q = 0; q < kRoBlocks; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][q][e][lane] = acc[q][e];
+  __syncthreads();
+  if ((lane & 15) >= n) return;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v = red[0][wave][e][lane];
+#pragma unroll
+    for (int i = 1; i < kRoWaves; ++i) v += red[i][wave][e][lane];
+    const int o = o0 + 16 * wave + 4 * (lane >> 4) + e;
+    if (o < options) logits[(int64_t)row * options + o] = bf16_to_f32(f32_to_bf16(v));
   }
 }
+
+static_assert(kRoBlocks == kRoWaves, "wave q stores block q");
 
 __global__ __launch_bounds__(64) void option_softmax_kernel(const float* __restrict__ logits, int32_t options,
                                                            const int32_t* __restrict__ adapters,
@@ -121,7 +164,7 @@ int launch_readout_logits(const uint16_t* hidden, int64_t hidden_stride, int32_t
   if (rows == 0) return MLORA_OK;
   const dim3 grid((unsigned)rows, (unsigned)((options + kRoOptionsPerBlock - 1) / kRoOptionsPerBlock));
   hipLaunchKernelGGL(readout_logits_kernel, grid, dim3(kRoThreads), 0, stream, hidden, hidden_stride, dim, pool,
-                     pool_stride, options, pool_rows, adapters, logits);
+                     pool_stride, options, pool_rows, adapters, rows, logits);
   return hipGetLastError() == hipSuccess ? MLORA_OK : MLORA_ELAUNCH;
 }
 
