@@ -8,6 +8,8 @@ import ctypes
 import threading
 from pathlib import Path
 
+import torch
+
 LIBRARY = Path(__file__).resolve().with_name("libjeff_mlora.so")
 ABI_VERSION = 2
 MAX_MATS = 8
@@ -133,6 +135,12 @@ def lib() -> ctypes.CDLL:
             raise LibraryMissing(f"{LIBRARY} has ABI version {version}; this package needs {ABI_VERSION} (rebuild)")
         _lib = h
         return h
+
+
+def stream_of(t: torch.Tensor) -> int:
+    """The current stream of t's GPU as a hipStream_t (torch.cuda.current_stream(t.device).cuda_stream without the
+    Stream object it makes)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def capture_id(stream: int) -> int:

@@ -38,7 +38,7 @@ def add_rms(x: torch.Tensor, d: torch.Tensor | None, w1: torch.Tensor) -> tuple[
         raise ValueError(f"add_rms: the row length must be a multiple of 8 up to {_lib.EPILOGUE_MAX_N}, got {n}")
     h = torch.empty(m, n, device=x.device, dtype=DT)
     xo = torch.empty(m, n, device=x.device, dtype=DT) if d is not None else x
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.stream_of(x)
     _lib.check(_lib.lib().mlora_add_rms(x.data_ptr(), x.stride(0), d.data_ptr() if d is not None else None,
                                         d.stride(0) if d is not None else 0, w1.data_ptr(),
                                         xo.data_ptr() if d is not None else None, xo.stride(0), h.data_ptr(),
@@ -60,7 +60,7 @@ def silu_mul(gu: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"silu_mul: the gate_up width must be twice a multiple of 8, got {width}")
     inter = width // 2
     y = torch.empty(rows, inter, device=gu.device, dtype=DT)
-    stream = torch.cuda.current_stream(gu.device).cuda_stream
+    stream = _lib.stream_of(gu)
     _lib.check(_lib.lib().mlora_silu_mul(gu.data_ptr(), gu.stride(0), y.data_ptr(), y.stride(0), rows, inter, stream),
                "mlora_silu_mul")
     return y

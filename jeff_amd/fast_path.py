@@ -94,6 +94,7 @@ class Lin:
         self.off_a = self.off_b = 0
         self.off_bj: list[int] = []
         self.int4: KernelInt4 | None = None
+        self._abi: _lib.Lora | None = None  # the last lora_abi, for the pool and rank table it describes
 
     def numel(self) -> int:
         """Pool elements per adapter row: A (rank, k) plus sB_j (out_j, cap_j) for every matrix."""
@@ -114,6 +115,7 @@ class Lin:
             ranks_table = torch.zeros(pool.shape[0], len(self.names), dtype=torch.int32, device=pool.device)
         self.ranks_table = ranks_table
         self.rank_col = rank_col
+        self._abi = None
 
     def pack(self, flat: torch.Tensor, updates: Mapping[str, Update]) -> list[int]:
         """Write one adapter's updates {matrix name: (A (r, in), sB (out, r))} into this group's slice of `flat` (all
@@ -140,14 +142,18 @@ class Lin:
         return live
 
     def lora_abi(self) -> _lib.Lora:
-        """The C description of this group's pool slice (pointers stay valid while the pool lives)."""
+        """The C description of this group's pool slice (pointers stay valid while the pool lives), made once per
+        binding."""
+        pool, table = self.pool.data_ptr(), self.ranks_table.data_ptr() + 4 * self.rank_col
+        if self._abi is not None and self._abi.pool == pool and self._abi.ranks == table:
+            return self._abi
         n = len(self.names)
         off_b = (_lib.c_i64 * _lib.MAX_MATS)(*(self.off_bj + [0] * (_lib.MAX_MATS - n)))
         cap = (_lib.c_i32 * _lib.MAX_MATS)(*(self.caps + [0] * (_lib.MAX_MATS - n)))
         cols = (_lib.c_i32 * _lib.MAX_MATS)(*(self.sizes + [0] * (_lib.MAX_MATS - n)))
-        ranks = self.ranks_table
-        return _lib.Lora(self.pool.data_ptr(), ranks.data_ptr() + 4 * self.rank_col, self.pool.stride(0), self.off_a,
-                         off_b, ranks.stride(0), self.pool.shape[0], n, self.rank, cap, cols)
+        self._abi = _lib.Lora(pool, table, self.pool.stride(0), self.off_a, off_b, self.ranks_table.stride(0),
+                              self.pool.shape[0], n, self.rank, cap, cols)
+        return self._abi
 
     def __call__(self, x: torch.Tensor, ws: Workspace, adp: torch.Tensor) -> torch.Tensor:
         """fast_path.py:347-349: the fused product of x through the bf16 W (torch's library GEMM) plus each token's
@@ -228,6 +234,10 @@ class Workspace:
         self.status = torch.zeros(1, **i32)
         self._last: RouteRecord | None = None
         self._route_abi: _lib.Route | None = None
+        # what every route of this workspace shares; a call's own sizes go into a copy
+        self._route_base = _lib.Route(self.req_order.data_ptr(), self.tok_perm.data_ptr(), self.last_of.data_ptr(),
+                                      self.seg_of.data_ptr(), self.seg_start.data_ptr(), self.seg_adapter.data_ptr(),
+                                      self.num_segs.data_ptr(), self.status.data_ptr(), 0, 0, 0)
         self._part: torch.Tensor | None = None
         self._retired: list[torch.Tensor] = []
         bound = max((h.mlora_int4_partials_bound(k, -(-out // 64) * 64, out, rows) for k, out in self.shapes),
@@ -272,12 +282,10 @@ class Workspace:
                 raise ValueError("cu_seqlens must be a contiguous int32 tensor of requests + 1 offsets")
         if tokens > self.rows:
             raise ValueError(f"A pass of {tokens} tokens does not fit a workspace of {self.rows}")
-        r = _lib.Route(self.req_order.data_ptr(), self.tok_perm.data_ptr(), self.last_of.data_ptr(),
-                       self.seg_of.data_ptr(), self.seg_start.data_ptr(), self.seg_adapter.data_ptr(),
-                       self.num_segs.data_ptr(), self.status.data_ptr(), tokens, requests,
-                       max(min(requests, pool_rows), 1))
+        r = _lib.Route.from_buffer_copy(self._route_base)
+        r.tokens, r.requests, r.max_segs = tokens, requests, max(min(requests, pool_rows), 1)
         h = _lib.lib()
-        stream = torch.cuda.current_stream(adp.device).cuda_stream
+        stream = _lib.stream_of(adp)
         _lib.check(h.mlora_route(adp.data_ptr(), 0 if cu_seqlens is None else cu_seqlens.data_ptr(),
                                  0 if cu_seqlens is not None else self.row_len, r, pool_rows, stream), "mlora_route")
         self._last = RouteRecord(weakref.ref(adp), adp._version, requests, tokens, pool_rows,
@@ -292,7 +300,7 @@ class Workspace:
         replays that launch before this product. Otherwise the route is launched again, with the cu_seqlens of the
         last ws.route of this adp when there was one (ragged rows), else over uniform rows of row_len."""
         last = self._last
-        stream = torch.cuda.current_stream(adp.device).cuda_stream
+        stream = _lib.stream_of(adp)
         capture = _lib.capture_id(stream)
         if last is not None and reusable(last, adp, tokens, pool_rows, stream, capture):
             return self._route_abi
@@ -331,7 +339,7 @@ def lora_add(y: torch.Tensor, x: torch.Tensor, lin: Lin, adp: torch.Tensor, ws: 
         raise ValueError(f"{', '.join(lin.names)}: stacked rank {lin.rank} exceeds the workspace's {ws.max_rank}")
     r = ws.routed(adp, lin.pool.shape[0], m)
     h = _lib.lib()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.stream_of(x)
     _lib.check(h.mlora_lora_add(lin.lora_abi(), r, x.data_ptr(), x.stride(0), lin.k, y.data_ptr(), y.stride(0),
                                 lin.out, ws.mid.data_ptr(), ws.mid.numel() * 2, flags, stream), "mlora_lora_add")
     return y

@@ -91,7 +91,7 @@ def int4_product(lin: Lin, x: torch.Tensor, ws: Workspace, adp: torch.Tensor, ti
     flags = (0 if tiles is None else tiles.flags()) | eflag
     w, lora = packed.abi(), lin.lora_abi()
     part, part_bytes = ws.partials(h.mlora_int4_partials_bytes(w, lora, r, flags))
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.stream_of(x)
     _lib.check(h.mlora_int4_linear(w, lora, r, x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0),
                                    0 if last_out is None else last_out.data_ptr(), ws.mid.data_ptr(),
                                    ws.mid.numel() * 2, part, part_bytes, flags, stream),
@@ -107,7 +107,7 @@ def shrink(lin: Lin, x: torch.Tensor, ws: Workspace, adp: torch.Tensor, mfma: bo
     r = ws.routed(adp, lin.pool.shape[0], m)
     flags = 0 if mfma is None else (_lib.FORCE_SHRINK_MFMA if mfma else _lib.FORCE_SHRINK_SEGMENT)
     h = _lib.lib()
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.stream_of(x)
     _lib.check(h.mlora_shrink(lin.lora_abi(), r, x.data_ptr(), x.stride(0), lin.k, ws.mid.data_ptr(), flags, stream),
                "mlora_shrink")
     return ws.mid[:m * lin.rank].view(m, lin.rank)
@@ -134,7 +134,7 @@ def base_expand(lin: Lin, x: torch.Tensor, ws: Workspace, adp: torch.Tensor, y: 
     flags = (0 if tiles is None else tiles.flags()) | eflag
     w, lora = packed.abi(), lin.lora_abi()
     part, part_bytes = ws.partials(h.mlora_int4_partials_bytes(w, lora, r, flags))
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = _lib.stream_of(x)
     _lib.check(h.mlora_int4_base_expand(w, lora, r, x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0),
                                         0 if last_out is None else last_out.data_ptr(), ws.mid.data_ptr(), part,
                                         part_bytes, flags, stream),

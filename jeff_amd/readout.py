@@ -47,7 +47,7 @@ def readout_logits(hidden: torch.Tensor, readout_pool: torch.Tensor, adapters: t
     _check_pool(hidden, readout_pool, "readout_logits")
     logits = torch.empty(b, readout_pool.shape[1], device=hidden.device, dtype=torch.float32)
     h = _lib.lib()
-    stream = torch.cuda.current_stream(hidden.device).cuda_stream
+    stream = _lib.stream_of(hidden)
     _lib.check(h.mlora_readout_logits(hidden.data_ptr(), hidden.stride(0), hidden.shape[1], readout_pool.data_ptr(),
                                       readout_pool.stride(0), readout_pool.shape[1], readout_pool.shape[0],
                                       adapters.data_ptr(), b, logits.data_ptr(), stream), "mlora_readout_logits")
@@ -71,7 +71,7 @@ def option_softmax(logits: torch.Tensor, adapters: torch.Tensor, counts: torch.T
                          f"{_lib.READOUT_MAX_OPTIONS} options, got {logits.dtype} {tuple(logits.shape)}")
     out = torch.empty_like(logits)
     h = _lib.lib()
-    stream = torch.cuda.current_stream(logits.device).cuda_stream
+    stream = _lib.stream_of(logits)
     _lib.check(h.mlora_option_softmax(logits.data_ptr(), logits.shape[1], adapters.data_ptr(), counts.data_ptr(),
                                       temp_pool.data_ptr(), temp_pool.shape[0], b, out.data_ptr(), stream),
                "mlora_option_softmax")
