@@ -204,7 +204,7 @@ size_t partials_of(const mlora_int4_t* w, const mlora_route_t* r, Base base, int
 // Whether a product of the family `base` runs as a sliced product (sliced.hip) instead of the family's own kernels. The
 // rule reads shapes only, never the epilogue, so a group's plain, gated and residual products sum in one order.
 //  - fused, long segments: when its estimate is below the 256 x 256 tiles' (a round of at most half the CUs: 19 us and
-//    0.94 a step; fuller: 1.4 a step), e.g. 384 rows of 2048 -> 2048, 6144 -> 2048 and 2048 -> 12288: 13, 24 and 38 us
+//    0.94 a step; fuller: 1.4 a step), e.g. 384 rows of 2048 -> 2048, 6144 -> 2048 and 2048 -> 12288: 16, 26 and 39 us
 //    against 45, 101 and 48; 2311 rows of 2048 -> 12288 stay on the tiles (131 us against 178);
 //  - split (short segments, 257 to 1023 rows): its segments' second factors in turn take about 1.8 us each, shared by the
 //    input slices, against the split product's range launch and epilogue: 643 rows of 128 adapters, 2048 -> 4096 and

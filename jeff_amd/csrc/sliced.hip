@@ -6,7 +6,7 @@
 // through LDS, rounded once and written (plain, added to the residual, or silu(gate) * up). Why this split: at these
 // sizes a product is a chain of latencies, not a stream. 256 x 256 tiles over all the inputs leave most CUs idle (384
 // rows of 2048 -> 2048: 16 tiles, 45 us); slicing the inputs inside the workgroup fills the CUs with short chains and
-// needs no float32 partials in memory and no second launch (13 us).
+// needs no float32 partials in memory and no second launch (16 us).
 //
 // What bounds it: the conversion of the packed weights (19 vector instructions a word of eight, RB MFMAs beside them), so
 // a step of 64 inputs a slice takes about 1.1 us whether RB is 1 or 3, plus 7 to 13 us of fixed time a round (launch,
@@ -227,7 +227,8 @@ __global__ __launch_bounds__(CW* KW * 64) void slice_kernel(mlora_int4_t w, mlor
 
   // Step i reads ring slot i % D and weight set i % D, in eight units e: the products of word e (16-input slice e / 2,
   // block e % 2) run while word e + 1 is dequantised and, at each even unit, the next slice's x operands are read. The
-  // step's barrier sits before its last slice: past it every wave has the step's last operands in registers, so the
+  // step's barrier sits before its last slice (a lone column wave needs none: it reads only what it staged, and the waves
+  // drift apart: 384 rows of 6144 -> 2048 30 -> 26 us): past it every wave has the step's last operands in registers, so the
   // slot takes step i + D's rows, and the next step's first operands are read while the last products run. Words are
   // loaded D steps ahead too, once the step's last word is converted. Loads complete in order; past the last step
   // they read nothing, so the number in flight at every wait stays the same.
@@ -248,8 +249,8 @@ __global__ __launch_bounds__(CW* KW * 64) void slice_kernel(mlora_int4_t w, mlor
       const int u = e >> 1, cb = e & 1;
       if (e == 6) {
         __builtin_amdgcn_sched_barrier(0);
-        MLORA_WAIT_VM((D - 2) * kXI + (D - 1) * kWI);  // x(i + 1) has landed
-        step_sync();
+        MLORA_WAIT_VM((D - 2) * kXI + (D - 1) * kWI);  // x(i + 1) has landed, and the step's operands are read
+        if constexpr (CW > 1) step_sync();             // (a lone column wave reads only the chunks it staged itself)
         dma_x(slot, i + D);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -482,13 +483,13 @@ __global__ __launch_bounds__(CW* KW * 64) void slice_kernel(mlora_int4_t w, mlor
 // takes a CU (its LDS): a round of them lasts a fixed time (launch, first loads, the sums' exchange and the stores) plus a
 // time per step, both measured on full rounds.
 SliceForm slice_form(int64_t tokens, int32_t columns, int32_t k, double* us) {
-  // measured with K = 2048 and 6144 over 384 and 2311 rows of 2048 to 12288 columns: 11.2 and 20.2 us a round,
-  // 12.9 and 23.5, 18.5 and 36.4, 35 and 78
+  // measured with K = 2048 and 6144 over 32, 384 and 2311 rows of 2048 to 12288 columns: 10.8 and 18.5 us a round,
+  // 15.6 and 25.6, 18.5 and 36.4, 35 and 78
   struct Cost {
     SliceForm f;
     double fixed, step;
   };
-  static const Cost costs[] = {{{1, 1, 8}, 6.7, 1.13}, {{2, 1, 8}, 7.6, 1.32}, {{2, 2, 4}, 9.5, 1.12}, {{3, 4, 2}, 13.5, 1.34}};
+  static const Cost costs[] = {{{1, 1, 8}, 7.0, 0.95}, {{2, 1, 8}, 10.6, 1.25}, {{2, 2, 4}, 9.5, 1.12}, {{3, 4, 2}, 13.5, 1.34}};
   const int cus = device_cus();
   SliceForm best = costs[0].f;
   double least = 0.0;
