@@ -274,7 +274,7 @@ def measure(name: str, steps: int, warmup: int, kernel_reps: int, headline: bool
                   "roofline": {"bound": "mfma", "achieved": step_flops / (ms_per_step / 1e3) / 1e12,
                                "peak": PEAK_BF16 / 1e12, "unit": "TFLOP/s",
                                "frac": step_flops / (ms_per_step / 1e3) / PEAK_BF16, "traffic": None,
-                               "kernel": "torch GEMM + lora_add (shrink_seg_kernel, base_mfma_kernel<false>)",
+                               "kernel": "torch GEMM + lora_add (first factors, lora_add_kernel)",
                                "note": "launch-bound: 0.55 GFLOP per step"},
                   "step_roofline": step_roof}
         del w, xs, keep, ws, last
@@ -331,8 +331,7 @@ def measure(name: str, steps: int, warmup: int, kernel_reps: int, headline: bool
     base, _, ranges = int4_plan(lin.int4.columns, lin.k, w.tokens, w.requests, pool_rows, lin.rank, lin.out,
                                 _lib.EPILOGUE_SILU_MUL if gated else 0)
     fin = " + silu(gate) * up" if gated else ""
-    kernel = {"mfma": f"base_mfma256_kernel (INT4 base + fused LoRA expand{fin})" if w.tokens >= 1024 or gated else
-              "base_mfma_kernel<true> (INT4 base + fused LoRA expand)",
+    kernel = {"mfma": f"base_mfma256_kernel (INT4 base + fused LoRA expand{fin})",
               "split": f"base_mfma256_kernel, split mode ({ranges} input ranges) + "
                        f"{'finish_gated_kernel' if gated else 'finish_kernel'} (INT4 base + LoRA expand{fin})",
               "narrow": (f"dec_kernel (INT4 base, {ranges} input ranges) + dec_expand_kernel (the ranges' sum + "

@@ -163,7 +163,9 @@ int mlora_route(const int32_t* adp, const int32_t* cu_seqlens, int32_t row_len, 
 /* The kernels mlora_int4_linear runs, without running them (host only, no GPU needed): for a pass of `tokens` tokens
  * in `requests` request rows over a pool of pool_rows rows, through a group of k inputs, `columns` kernel columns,
  * `out` outputs and rank_cap stacked ranks, with these flags. *base: 0 the GEMV (at most 8 tokens), 1 the MFMA tile
- * kernel with the second factor fused, 2 the split product, 3 the narrow product; *shrink: 0 the segment form, 1
+ * kernel with the second factor fused, 2 the split product, 3 the narrow product (1 to 3 are families: within them the
+ * sliced product, one launch with the inputs sliced over a workgroup's waves, runs where it is estimated faster; it reads
+ * no partials); *shrink: 0 the segment form, 1
  * the MFMA form of the first factor; *ranges: input ranges of a split or narrow product (1 otherwise; the narrow
  * count depends on the current device's CU count, 256 without a device). MLORA_EUNSUPPORTED as mlora_int4_linear
  * would return it for forced flags that cannot run. */

@@ -2,9 +2,10 @@
 //   y[perm[p], c] = bf16( sum_k x[perm[p], k] W[c, k]  +  sum_q mid[p, rho_j + q] sB_j[a][c - o_j, q] )
 // W[c, k] = bf16((code - z) s) is dequantised in registers from the packed words; the base and the LoRA term are
 // accumulated in float32 and rounded once (the reference's cut product, engine/int4_kernels.py:105-129, without its
-// float32 partial buffer). Without the base (kBase = false) the kernels compute lora_add: y += the LoRA term, in place
-// (engine/fast_path.py:180-203,277-289).
-//  - base_mfma: tiles of 128 sorted tokens x 128 columns, 4 waves of 64 x 64, 32x32x16 bf16 MFMA. Each K step of 64
+// float32 partial buffer). lora_add (y += the LoRA term, in place, engine/fast_path.py:180-203,277-289) is the GEMV kernel
+// without the base (kBase = false) up to 8 tokens and lora_add_kernel past them.
+//  - base_mfma: the passes whose rows' 32-bit element offsets do not fit (the others take the 256 x 256 tiles, the sliced
+//    or the decode products): tiles of 128 sorted tokens x 128 columns, 4 waves of 64 x 64, 32x32x16 bf16 MFMA. Each K step of 64
 //    stages x (gathered through the sorted order) and the dequantised weights through LDS; the next step's words and
 //    activations are fetched into registers while the MFMAs run.
 //  - base_gemv: at most 8 tokens (decode of a few rows). 64 input slices x 16 columns per workgroup, x staged in LDS

@@ -1,6 +1,6 @@
 // Adapter routing: request rows -> segments of the sorted order, one segment per adapter present.
 // Replaces the reference's per-tile lookup adp[t // row_len] (engine/fast_path.py:167,189;
-// engine/int4_kernels.py:72,113) with a stable sort, so every adapter's tokens are contiguous.
+// engine/int4_kernels.py:72,113) with a stable order, so every adapter's tokens are contiguous.
 #include "mlora_common.h"
 
 namespace {

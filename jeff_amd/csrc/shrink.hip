@@ -1,10 +1,12 @@
 // The LoRA first factor ("shrink"): mid[p, rho_j + q] = bf16( sum_k x[perm[p], k] A_j[a][q, k] ) for every sorted
 // token position p of an adapter segment, matrix j of the group and live rank q. Summed in float32 in a fixed
 // order and rounded once to bf16, as the reference rounds its first factor before the second product
-// (engine/fast_path.py:159-177,196; engine/int4_kernels.py:67-82,120). Two kernels, chosen by segment length:
+// (engine/fast_path.py:159-177,196; engine/int4_kernels.py:67-82,120). Three kernels, chosen by segment length and size:
 //  - shrink_seg: few tokens per adapter (decode). One workgroup per (segment, 32-rank block) streams those 32 rows
 //    of A once into MFMA operands, the segment's rows as the other operand; its waves split the inputs and add their
 //    sums in a fixed order. Memory-bound on A.
+//  - shrink_rows: long segments, few rows. One workgroup per 32 sorted rows and 32 stacked ranks, the inputs sliced over
+//    its 16 waves.
 //  - shrink_tile: long segments (prefill). Workgroups per 128 sorted positions, 4 waves of 32 rows; the x rows and
 //    the adapter's A rows stream through LDS rings two steps ahead, A shared by the waves; each wave sums its rows
 //    over all the inputs in order.

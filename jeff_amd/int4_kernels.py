@@ -6,7 +6,8 @@ input that is not a contiguous bf16 (tokens, lin.k) tensor, or a pass too large 
 stream: the LoRA first factor, then either the base product with the second factor fused into its epilogue (one
 launch, rounded once) or, for passes with few tokens per adapter (decode), the reference's split product: float32
 partial products over ranges of the input dimension, then one epilogue launch per (adapter segment, 256 columns)
-that adds them in order with the LoRA term and rounds once. Plus the routing launch when the workspace has not
+that adds them in order with the LoRA term and rounds once. Small and medium passes of either kind run the sliced product
+(one launch, no partials) where it is the faster. Plus the routing launch when the workspace has not
 routed `adp` yet. Deterministic: no atomic additions, every sum in a fixed order."""
 
 from __future__ import annotations

@@ -9,9 +9,11 @@ call that needs no GPU, so the kernel a benchmark names is the one the product r
   dimension split into float32 ranges only when the columns are too few for the CUs) or "split" (few tokens per
   segment, more tokens: MFMA tiles over ranges of the input dimension into float32 partials, then one epilogue
   workgroup per adapter segment and 256 columns).
+Within "mfma" (long segments), "split" and "narrow" the library runs the sliced product (csrc/sliced.hip: tiles of 32 to
+96 rows, the inputs sliced over a workgroup's waves) where its estimate is the lower one; the family's name stays.
 - shrink (the LoRA first factor): "segment" when segments are short on average (decode: one workgroup per segment
   and 32 ranks of its adapter's A, the segment's rows as the second MFMA operand) or "mfma" when they are long
-  (prefill: 32 sorted rows per workgroup on MFMA)."""
+  (prefill: 32 or 128 sorted rows per workgroup on MFMA)."""
 
 from __future__ import annotations
 
