@@ -11,10 +11,9 @@ namespace {
 
 using namespace mlora;
 
-constexpr int kRmsRows = 4;                          // rows (waves) per workgroup
+constexpr int kRmsRows = 4;                             // rows (waves) per workgroup
 constexpr int kRmsChunks = MLORA_EPILOGUE_MAX_N / 512;  // 16-byte chunks per lane at the largest row
-constexpr int kRmsGroup = 2;                            // chunks per lane whose loads are issued together
-static_assert(kRmsChunks % kRmsGroup == 0, "whole groups of chunks");
+constexpr int kRmsShort = 4;                            // the same of a short row (up to 2048 inputs)
 
 __device__ __forceinline__ float wave_sum_fixed(float v) {
 #pragma unroll
@@ -22,35 +21,55 @@ __device__ __forceinline__ float wave_sum_fixed(float v) {
   return v;
 }
 
+// CH: the chunks per lane a row may have. A short row asks for all it reads at once, the weights among them (a few rows
+// are one chain of latencies: the row, the wave's sum, the weights; 4 rows of 2048 3.9 -> 3.2 us, 384 rows 4.5 -> 3.7), and
+// its registers leave many waves in flight where memory bounds it (159488 rows of 2048 465 -> 458 us, 5.7 TB/s). Rows past
+// that keep two chunks in flight: their weights asked for with the row cost a wave a SIMD (20000 rows of 8192 261 -> 299).
+template <int CH>
 __global__ __launch_bounds__(kRmsRows * 64) void add_rms_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
                                                                 const uint16_t* __restrict__ d, int64_t d_stride,
                                                                 const float* __restrict__ w1,
                                                                 uint16_t* __restrict__ xo, int64_t xo_stride,
                                                                 uint16_t* __restrict__ h, int64_t h_stride,
                                                                 int64_t rows, int32_t n, float eps) {
+  constexpr bool kAhead = CH <= kRmsShort;  // the weights are asked for with the row
+  constexpr int kGroup = kAhead ? CH : 2;   // chunks per lane whose loads are issued together
+  static_assert(CH % kGroup == 0, "whole groups of chunks");
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kRmsRows + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int chunks = n / 8;
   const uint16_t* xr = x + row * x_stride;
-  float v[kRmsChunks][8];
+  float v[CH][8];
   float ss = 0.0f;
-  // The lane's chunks are taken kRmsGroup at a time: the group's x and d loads are all issued before the first is
+  float4 w_lo[kGroup], w_hi[kGroup];
+  auto load_w = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kGroup; ++u) {
+      const int c = lane + 64 * (i0 + u);
+      if (c < chunks) {
+        w_lo[u] = *reinterpret_cast<const float4*>(w1 + 8 * c);
+        w_hi[u] = *reinterpret_cast<const float4*>(w1 + 8 * c + 4);
+      }
+    }
+  };
+  // The lane's chunks are taken kGroup at a time: the group's x and d loads are all issued before the first is
   // used (one memory latency per group, not two per chunk); the sums run in chunk order as before.
 #pragma unroll
-  for (int i0 = 0; i0 < kRmsChunks; i0 += kRmsGroup) {
+  for (int i0 = 0; i0 < CH; i0 += kGroup) {
     if (lane + 64 * i0 >= chunks) break;
-    uint4 xv[kRmsGroup], dv[kRmsGroup];
+    uint4 xv[kGroup], dv[kGroup];
 #pragma unroll
-    for (int u = 0; u < kRmsGroup; ++u) {
+    for (int u = 0; u < kGroup; ++u) {
       const int c = lane + 64 * (i0 + u);
       if (c < chunks) {
         xv[u] = *reinterpret_cast<const uint4*>(xr + 8 * c);
         if (d != nullptr) dv[u] = *reinterpret_cast<const uint4*>(d + row * d_stride + 8 * c);
       }
     }
+    if constexpr (kAhead) load_w(i0);
 #pragma unroll
-    for (int u = 0; u < kRmsGroup; ++u) {
+    for (int u = 0; u < kGroup; ++u) {
       const int i = i0 + u, c = lane + 64 * i;
       if (c >= chunks) break;
       const uint32_t xw[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
@@ -75,22 +94,14 @@ __global__ __launch_bounds__(kRmsRows * 64) void add_rms_kernel(const uint16_t* 
   ss = wave_sum_fixed(ss);
   const float r = 1.0f / __builtin_sqrtf(ss / (float)n + eps);
 #pragma unroll
-  for (int i0 = 0; i0 < kRmsChunks; i0 += kRmsGroup) {
+  for (int i0 = 0; i0 < CH; i0 += kGroup) {
     if (lane + 64 * i0 >= chunks) break;
-    float4 wa[kRmsGroup], wb[kRmsGroup];
+    if constexpr (!kAhead) load_w(i0);
 #pragma unroll
-    for (int u = 0; u < kRmsGroup; ++u) {
-      const int c = lane + 64 * (i0 + u);
-      if (c < chunks) {
-        wa[u] = *reinterpret_cast<const float4*>(w1 + 8 * c);
-        wb[u] = *reinterpret_cast<const float4*>(w1 + 8 * c + 4);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kRmsGroup; ++u) {
+    for (int u = 0; u < kGroup; ++u) {
       const int i = i0 + u, c = lane + 64 * i;
       if (c >= chunks) break;
-      const float wv[8] = {wa[u].x, wa[u].y, wa[u].z, wa[u].w, wb[u].x, wb[u].y, wb[u].z, wb[u].w};
+      const float wv[8] = {w_lo[u].x, w_lo[u].y, w_lo[u].z, w_lo[u].w, w_hi[u].x, w_hi[u].y, w_hi[u].z, w_hi[u].w};
       uint32_t hw[4];
 #pragma unroll
       for (int e = 0; e < 8; e += 2) hw[e >> 1] = pack_bf16x2(v[i][e] * r * wv[e], v[i][e + 1] * r * wv[e + 1]);
@@ -120,8 +131,12 @@ int launch_add_rms(const uint16_t* x, int64_t x_stride, const uint16_t* d, int64
                    hipStream_t stream) {
   if (rows == 0) return MLORA_OK;
   const int64_t blocks = (rows + kRmsRows - 1) / kRmsRows;
-  hipLaunchKernelGGL(add_rms_kernel, dim3((unsigned)blocks), dim3(kRmsRows * 64), 0, stream, x, x_stride, d, d_stride,
-                     w1, xo, xo_stride, h, h_stride, rows, n, eps);
+  // (up to 1024 inputs half of kRmsShort's chunks: 384 rows of 1024 3.2 -> 2.9 us, 159488 rows 221 -> 224 against 227)
+  auto kernel = n <= 256 * kRmsShort   ? add_rms_kernel<kRmsShort / 2>
+                : n <= 512 * kRmsShort ? add_rms_kernel<kRmsShort>
+                                       : add_rms_kernel<kRmsChunks>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kRmsRows * 64), 0, stream, x, x_stride, d, d_stride, w1, xo,
+                     xo_stride, h, h_stride, rows, n, eps);
   return hipGetLastError() == hipSuccess ? MLORA_OK : MLORA_ELAUNCH;
 }
 

@@ -54,6 +54,16 @@ def test_add_rms(rows: int, n: int) -> None:
     torch.testing.assert_close(h.float(), want.float(), rtol=BF16_STEP, atol=1e-6)
 
 
+@pytest.mark.parametrize("rows,n", [(5, 1016), (5, 1032), (6, 2040), (6, 2056)])
+def test_add_rms_at_the_edges_of_its_row_lengths(rows: int, n: int) -> None:
+    """Around 1024 and 2048 inputs, where the row's registers change: x + d exact, h within a bfloat16 step."""
+    x, d, w1 = case(rows, n, rows + n)
+    xo, h = add_rms(x, d, w1)
+    xo_bits, h_exact, h_bits = oracle_add_rms(bits(x), bits(d), w1.cpu().numpy())
+    assert np.array_equal(bits(xo), xo_bits)
+    check_close(h, h_exact, h_bits, "add_rms h")
+
+
 def test_rms_without_residual_returns_x_itself() -> None:
     x, _, w1 = case(33, 2048, 3)
     xo, h = add_rms(x, None, w1)
