@@ -242,6 +242,10 @@ int run_base(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* 
              void* partials, size_t partials_bytes, Base base, int32_t flags, hipStream_t s) {
   const int32_t inter = gated_width(w, flags);
   const bool resid = residual_of(flags);
+  // (a split product's partials are asked for whichever kernels run it: the caller knows the family, not the kernels)
+  if (base == Base::split &&
+      (partials == nullptr || !aligned16(partials) || partials_bytes < split_bytes(w, r->tokens)))
+    return MLORA_EWORKSPACE;
   if (use_slice(w, L, r, x_stride, base, flags)) {
     if (fuse_shrink) {
       const int rc = launch_shrink(*L, *r, x, x_stride, w->k, mid, false, s);
@@ -260,8 +264,6 @@ int run_base(const mlora_int4_t* w, const mlora_lora_t* L, const mlora_route_t* 
     return launch_base256(*w, *L, *r, x, x_stride, y, y_stride, last_out, w->out, mid, nullptr, 1, s, inter, resid);
   if (base != Base::split)
     return launch_base(w, *L, *r, x, x_stride, y, y_stride, last_out, w->out, mid, base == Base::gemv, s);
-  if (partials == nullptr || !aligned16(partials) || partials_bytes < split_bytes(w, r->tokens))
-    return MLORA_EWORKSPACE;
   const int32_t ks = split_ranges(w, r->tokens);
   float* part = static_cast<float*>(partials);
   int rc = launch_base256(*w, *L, *r, x, x_stride, nullptr, 0, nullptr, w->out, nullptr, part, ks, s);
@@ -431,9 +433,9 @@ int mlora_int4_linear(const mlora_int4_t* w, const mlora_lora_t* lora, const mlo
   if (workspace_bytes < mlora_workspace_bytes(route->tokens, lora->rank_cap)) return MLORA_EWORKSPACE;
   Base base;
   if ((rc = base_of(w, lora, route, x_stride, flags, &base))) return rc;
-  const bool sliced = use_slice(w, lora, route, x_stride, base, flags);
-  if (base == Base::split && !sliced && (partials == nullptr || partials_bytes < split_bytes(w, route->tokens)))
+  if (base == Base::split && (partials == nullptr || partials_bytes < split_bytes(w, route->tokens)))
     return MLORA_EWORKSPACE;
+  const bool sliced = use_slice(w, lora, route, x_stride, base, flags);
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint16_t* mid = static_cast<uint16_t*>(workspace);
   const bool mfma_shrink = shrink_on_mfma(route, lora->pool_rows, flags);

@@ -112,3 +112,25 @@ def test_first_factor_extent_past_32_bits_is_refused() -> None:
     assert h.mlora_shrink(ctypes.byref(lora), ctypes.byref(r), 16, 64, 64, 16, 0, None) == _lib.EOVERFLOW
     assert h.mlora_int4_base_expand(ctypes.byref(w), ctypes.byref(lora), ctypes.byref(r), 16, 64, 16, 64, None, 16,
                                     None, 0, 0, None) == _lib.EOVERFLOW
+
+
+def test_split_product_without_its_partials_is_refused() -> None:
+    """A split product (643 rows of 128 adapters) asks for its float32 partials whichever kernels run it: without them,
+    or with one byte too few, it is refused with MLORA_EWORKSPACE before any launch."""
+    h = _lib.lib()
+    k, n, rank, tokens = 2048, 2048, 16, 643
+    mats = (_lib.c_i64 * _lib.MAX_MATS)(rank * k, *([0] * (_lib.MAX_MATS - 1)))
+    caps = (_lib.c_i32 * _lib.MAX_MATS)(rank, *([0] * (_lib.MAX_MATS - 1)))
+    cols = (_lib.c_i32 * _lib.MAX_MATS)(n, *([0] * (_lib.MAX_MATS - 1)))
+    lora = _lib.Lora(16, 16, rank * (k + n), 0, mats, 1, 129, 1, rank, caps, cols)
+    w = _lib.Int4(16, 16, None, k, n, n, 64)
+    r = _lib.Route(16, 16, 16, 16, 16, 16, 16, 16, tokens, tokens, 129)
+    base, shrink, ranges = (ctypes.c_int32() for _ in range(3))
+    assert h.mlora_int4_plan(k, n, n, tokens, tokens, 129, rank, 0, ctypes.byref(base), ctypes.byref(shrink),
+                             ctypes.byref(ranges)) == 0
+    need = ranges.value * tokens * n * 4
+    for partials, size in ((None, 1 << 40), (16, need - 1)):
+        assert h.mlora_int4_linear(ctypes.byref(w), ctypes.byref(lora), ctypes.byref(r), 16, k, 16, n, None, 16,
+                                   1 << 40, partials, size, 0, None) == _lib.EWORKSPACE
+        assert h.mlora_int4_base_expand(ctypes.byref(w), ctypes.byref(lora), ctypes.byref(r), 16, k, 16, n, None, 16,
+                                        partials, size, 0, None) == _lib.EWORKSPACE
