@@ -94,7 +94,7 @@ class Lin:
         self.off_a = self.off_b = 0
         self.off_bj: list[int] = []
         self.int4: KernelInt4 | None = None
-        self._abi: _lib.Lora | None = None  # the last lora_abi, for the pool and rank table it describes
+        self._layout: _lib.Lora | None = None  # the binding's offsets, widths and capacities (no pointers)
 
     def numel(self) -> int:
         """Pool elements per adapter row: A (rank, k) plus sB_j (out_j, cap_j) for every matrix."""
@@ -115,7 +115,9 @@ class Lin:
             ranks_table = torch.zeros(pool.shape[0], len(self.names), dtype=torch.int32, device=pool.device)
         self.ranks_table = ranks_table
         self.rank_col = rank_col
-        self._abi = None
+        n = len(self.names)
+        self._layout = _lib.Lora(None, None, 0, offset, (_lib.c_i64 * _lib.MAX_MATS)(*self.off_bj), 0, 0, n, self.rank,
+                                 (_lib.c_i32 * _lib.MAX_MATS)(*self.caps), (_lib.c_i32 * _lib.MAX_MATS)(*self.sizes))
 
     def pack(self, flat: torch.Tensor, updates: Mapping[str, Update]) -> list[int]:
         """Write one adapter's updates {matrix name: (A (r, in), sB (out, r))} into this group's slice of `flat` (all
@@ -142,18 +144,13 @@ class Lin:
         return live
 
     def lora_abi(self) -> _lib.Lora:
-        """The C description of this group's pool slice (pointers stay valid while the pool lives), made once per
-        binding."""
-        pool, table = self.pool.data_ptr(), self.ranks_table.data_ptr() + 4 * self.rank_col
-        if self._abi is not None and self._abi.pool == pool and self._abi.ranks == table:
-            return self._abi
-        n = len(self.names)
-        off_b = (_lib.c_i64 * _lib.MAX_MATS)(*(self.off_bj + [0] * (_lib.MAX_MATS - n)))
-        cap = (_lib.c_i32 * _lib.MAX_MATS)(*(self.caps + [0] * (_lib.MAX_MATS - n)))
-        cols = (_lib.c_i32 * _lib.MAX_MATS)(*(self.sizes + [0] * (_lib.MAX_MATS - n)))
-        self._abi = _lib.Lora(pool, table, self.pool.stride(0), self.off_a, off_b, self.ranks_table.stride(0),
-                              self.pool.shape[0], n, self.rank, cap, cols)
-        return self._abi
+        """The C description of this group's pool slice as it is now (pointers stay valid while the pool lives): the
+        binding's layout with the pool's and the rank table's pointers, rows and strides."""
+        r = _lib.Lora.from_buffer_copy(self._layout)
+        r.pool, r.pool_stride = self.pool.data_ptr(), self.pool.stride(0)
+        r.ranks, r.ranks_stride = self.ranks_table.data_ptr() + 4 * self.rank_col, self.ranks_table.stride(0)
+        r.pool_rows = self.pool.shape[0]
+        return r
 
     def __call__(self, x: torch.Tensor, ws: Workspace, adp: torch.Tensor) -> torch.Tensor:
         """fast_path.py:347-349: the fused product of x through the bf16 W (torch's library GEMM) plus each token's

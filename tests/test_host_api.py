@@ -235,3 +235,18 @@ def test_partials_bound_covers_every_automatic_product() -> None:
                     assert bound >= need, (k, out, tokens, t, requests, base, ranges, need, bound)
     assert h.mlora_int4_partials_bound(100, 64, 64, 8) == 0
     assert h.mlora_int4_partials_bound(2048, 4096, 4096, 0) == 0
+
+
+def test_a_groups_description_follows_the_pool_it_is_bound_to() -> None:
+    """The C description reads the pool and rank table as they are at the call: a view of fewer rows at the same
+    address, or another pool, is described by its own rows, strides and pointers."""
+    lin = Lin(["l.q_proj", "l.k_proj"], sizes=[24, 16], k=32, ranks=[16, 8])
+    AdapterPool([lin], 6, device="cpu")
+    first = lin.lora_abi()
+    assert first.pool_rows == 7 and list(first.off_b)[:2] == lin.off_bj and list(first.cap)[:2] == [16, 8]
+    lin.pool = lin.pool[:3]
+    assert lin.lora_abi().pool_rows == 3 and lin.lora_abi().pool == first.pool
+    lin.pool = torch.zeros(5, 2 * lin.numel(), dtype=DT)[:, :lin.numel()]
+    got = lin.lora_abi()
+    assert (got.pool, got.pool_rows, got.pool_stride) == (lin.pool.data_ptr(), 5, 2 * lin.numel())
+    assert first.pool_rows == 7  # a description handed out stays as it was
