@@ -139,7 +139,9 @@ def lib() -> ctypes.CDLL:
 
 def stream_of(t: torch.Tensor) -> int:
     """The current stream of t's GPU as a hipStream_t (torch.cuda.current_stream(t.device).cuda_stream without the
-    Stream object it makes)."""
+    Stream object it makes); ValueError for a tensor that is on no GPU, as there."""
+    if not t.is_cuda:
+        raise ValueError(f"Expected a cuda device, but got: {t.device}")
     return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 

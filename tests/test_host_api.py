@@ -7,6 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from jeff_amd import _lib
 from jeff_amd.fast_path import DT, AdapterPool, Lin, Workspace, fold_scale, sb_stride
 from jeff_amd.int4 import Int4Error, pack_kernel, pack_kernel_asym, unpack_kernel, unpack_kernel_asym
 from jeff_amd.int4_kernels import int4_product
@@ -250,3 +251,8 @@ def test_a_groups_description_follows_the_pool_it_is_bound_to() -> None:
     got = lin.lora_abi()
     assert (got.pool, got.pool_rows, got.pool_stride) == (lin.pool.data_ptr(), 5, 2 * lin.numel())
     assert first.pool_rows == 7  # a description handed out stays as it was
+
+
+def test_a_tensor_off_the_gpu_has_no_stream() -> None:
+    with pytest.raises(ValueError, match="cuda"):
+        _lib.stream_of(torch.zeros(1))
