@@ -50,8 +50,13 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(const int32_t* __r
   bool bad_adapter = false;
   for (int i = tid; i < B; i += kRouteThreads) {
     int a = adp[i];
-    const int len = cu != nullptr ? cu[i + 1] - cu[i] : row_len;
-    bad |= len < 0;
+    // (offsets are compared, not subtracted: two more than 2^31 apart differ by a wrapped length of either sign)
+    int len = row_len;
+    if (cu != nullptr) {
+      const int c0 = cu[i], c1 = cu[i + 1];
+      bad |= c1 < c0;
+      len = c1 < c0 ? 0 : (int)((uint32_t)c1 - (uint32_t)c0);
+    }
     if (a < 0 || a >= pool_rows) {
       a = 0;
       bad_adapter = true;

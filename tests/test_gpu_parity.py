@@ -119,6 +119,19 @@ def test_route_flags_unusable_seqlens_and_falls_back_to_identity(cu: list) -> No
         ws.check()
 
 
+@pytest.mark.parametrize("at,values", [(0, [1]), (10, [7]), (68, [400]), (69, [211]),
+                                       (10, [2_000_000_000, -2_000_000_000])])  # whose difference wraps to a length
+def test_route_of_many_requests_flags_unusable_seqlens(at: int, values: list) -> None:
+    """More than 64 requests (a workgroup per 32): offsets that start past 0 or decrease anywhere, by however much."""
+    cu = 3 * np.arange(71)
+    cu[at:at + len(values)] = values
+    ws, tokens = run_route(np.arange(70) % 4, 4, None, cu)
+    assert tokens == 210 and int(ws.status.item()) == _lib.ROUTE_BAD_SEQLENS
+    assert np.array_equal(ws.tok_perm[:tokens].cpu().numpy(), np.arange(tokens))
+    assert not ws.seg_of[:tokens].cpu().numpy().any()
+    assert int(ws.num_segs.item()) == 1 and int(ws.seg_adapter[0].item()) == 0
+
+
 @pytest.mark.parametrize("group,asym", [(64, False), (128, False), (64, True), (128, True)])
 def test_dequant_is_bit_exact(group: int, asym: bool) -> None:
     g = torch.Generator().manual_seed(group + asym)
